@@ -214,44 +214,36 @@ bool latency_config(int64_t rows, int64_t nvec, int mode, hprms_config* c) {
   return false;
 }
 
-// The FP8 output adds a second row reduction (the absolute maximum) and a
-// barrier; at 1K < H <= 2K it prefers two vectors per lane, one row per
-// 128-lane workgroup (5-9% faster than the fused table's 64 x 4 at 4096 rows,
-// as for the MX outputs, 5-11%); from 3K elements more, smaller workgroups per CU, and
-// at 32K the LDS tier (measured 5.8% faster than 1024 lanes x 4 in registers),
-// with the residual's loads first (1-1.9% faster at 25K-32K).
-bool fp8_config(int64_t nvec, hprms_config* c) {
-  struct Row { int64_t min_nvec, max_nvec; int lpr, vpl, ldsv, block, flags; };
-  static const Row fp8[] = {{129, 256, 128, 2, 0, 128, 3},
-                            {385, 512, 256, 2, 0, 256, 7},
-                            {513, 640, 256, 3, 0, 256, 7},
-                            {641, 1024, 512, 2, 0, 512, 7},
-                            {1537, 2048, 1024, 2, 0, 1024, 31},
-                            {3073, 4096, 512, 8, 4, 512, 159}};
-  for (const Row& r : fp8) {
-    if (nvec >= r.min_nvec && nvec <= r.max_nvec) {
+// The quantised outputs (FP8: a second row reduction and a barrier; MX and FP8
+// per 128 elements: per-block maxima by DPP) prefer two vectors per lane, one
+// row per 128-lane workgroup, at 1K < H <= 2K (5-11% faster than the fused
+// table's 64 x 4 at 4096 rows), 256 lanes x 2 at 3K < H <= 4K, and from 12K
+// on workgroups of 256 and 512 lanes with more vectors each rather than 1024
+// lanes: more workgroups stand on a CU, so the barriers of one hide behind
+// the loads of others.  Against 1024 x 2 at 16384 (bf16; per-row FP8, MXFP4):
+// 512 rows 13.7 -> 11.9 us and 12.4 -> 10.8 us, 4096 rows 83.0 -> 78.8 us and
+// 75.3 -> 71.6 us; 512 x 5-6 against 1024 x 3: per-row FP8 11-30% faster at
+// 20K-24K from 1 to 4096 rows, MXFP4 4-23% up to 768 rows and within 2% at
+// 4096.  Past 24K the LDS tier (per row) and 1024 x 4 (per block) stay, 2-5%
+// ahead of 512 x 8 in registers.  256 x 8 against 512 x 4 at 16384: MXFP4
+// 2-4% and FP8 per 128 elements 2% faster, per-row FP8 the same.
+bool quant_config(int64_t nvec, int mode, hprms_config* c) {
+  struct Row { unsigned modes; int64_t min_nvec, max_nvec; int lpr, vpl, ldsv, block, flags; };
+  constexpr unsigned all = ~0u, row = 1u << 2, blocks = ~row;
+  static const Row quant[] = {{all, 129, 256, 128, 2, 0, 128, 3},
+                              {all, 385, 512, 256, 2, 0, 256, 7},
+                              {all, 513, 640, 256, 3, 0, 256, 7},
+                              {all, 641, 1024, 512, 2, 0, 512, 7},
+                              {row, 1537, 2048, 512, 4, 0, 512, 7},
+                              {blocks, 1537, 1792, 512, 4, 0, 512, 7},
+                              {blocks, 1793, 2048, 256, 8, 0, 256, 7},
+                              {all, 2049, 2560, 512, 5, 0, 512, 135},
+                              {all, 2561, 3072, 512, 6, 0, 512, 135},
+                              {row, 3073, 4096, 512, 8, 4, 512, 159},
+                              {blocks, 3073, 4096, 1024, 4, 0, 1024, 159}};
+  for (const Row& r : quant) {
+    if (((r.modes >> mode) & 1u) && nvec >= r.min_nvec && nvec <= r.max_nvec) {
       *c = hprms_config{r.ldsv > 0 ? 2 : 1, r.lpr, r.vpl, r.ldsv, r.block, 0, r.flags};
-      return true;
-    }
-  }
-  return false;
-}
-
-// The MX outputs (per-block maxima: a DPP quad step, no second barrier)
-// measured best with the register tier at 32K (1024 x 4: 4.5% / 5% faster
-// than the FP8 table's LDS tier for MXFP8 / MXFP4) and with 256 lanes x 2 at
-// 3K < H <= 4K.
-bool mx_config(int64_t nvec, hprms_config* c) {
-  struct Row { int64_t min_nvec, max_nvec; int lpr, vpl, ldsv, block, flags; };
-  static const Row mx[] = {{129, 256, 128, 2, 0, 128, 3},
-                           {385, 512, 256, 2, 0, 256, 7},
-                           {513, 640, 256, 3, 0, 256, 7},
-                           {641, 1024, 512, 2, 0, 512, 7},
-                           {1537, 2048, 1024, 2, 0, 1024, 31},
-                           {3073, 4096, 1024, 4, 0, 1024, 159}};
-  for (const Row& r : mx) {
-    if (nvec >= r.min_nvec && nvec <= r.max_nvec) {
-      *c = hprms_config{1, r.lpr, r.vpl, r.ldsv, r.block, 0, r.flags};
       return true;
     }
   }
@@ -400,8 +392,7 @@ void table_config(int64_t rows, int64_t hidden, int mode, bool grid, int cus, hp
   if (mode == 0 && grid && inplace_config(nvec, c)) return;
   if (mode == 1 && plain_config(nvec, c)) return;
   if (mode == 4 && reduce_config(nvec, c)) return;
-  if (mode == 2 && fp8_config(nvec, c)) return;
-  if (mode >= 5 && mx_config(nvec, c)) return;   // MX and the FP8 output with a scale per 128 elements
+  if ((mode == 2 || mode >= 5) && quant_config(nvec, mode, c)) return;
   *c = hprms_config{1, 0, 0, 0, 0, 0, 3};
   // flags: 3 = non-temporal row loads and stores, +4 = weight loaded late,
   // +24 = sc1 on loads and stores, +128 = residual loads before input loads

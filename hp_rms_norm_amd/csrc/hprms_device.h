@@ -14,6 +14,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+#include <utility>
+
 #include "hp_rms_norm_amd.h"
 
 namespace hprms {
@@ -54,6 +57,17 @@ template <typename T>
 __device__ __forceinline__ T opaque(T v) {
   asm volatile("" : "+s"(v));
   return v;
+}
+
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>): an
+// unrolled loop whose index is a constant expression (DPP controls).
+template <class Fn, int... K>
+__device__ __forceinline__ void each_of(std::integer_sequence<int, K...>, Fn&& f) {
+  (f(std::integral_constant<int, K>{}), ...);
+}
+template <int N, class Fn>
+__device__ __forceinline__ void each(Fn&& f) {
+  each_of(std::make_integer_sequence<int, N>{}, f);
 }
 
 // ---- element formats --------------------------------------------------------
@@ -113,9 +127,16 @@ __device__ __forceinline__ uint32_t pack_e4m3x4(float a, float b, float c, float
   return (uint32_t)w;
 }
 
-// Clamp to the e4m3fn range; NaN passes through (both compares are false).
+// Clamp to the e4m3fn range; NaN passes through (IEEE 754-2019 minimum and
+// maximum, one gfx950 instruction each; compares and selects took four).
 __device__ __forceinline__ float clamp_e4m3(float v) {
-  return v > 448.0f ? 448.0f : (v < -448.0f ? -448.0f : v);
+  return __builtin_elementwise_minimum(__builtin_elementwise_maximum(v, -448.0f), 448.0f);
+}
+
+// The four e4m3fn bytes of w with an overflowed code (0x7f, either sign), as
+// the conversions give it past 464, replaced by the largest finite one (0x7e).
+__device__ __forceinline__ uint32_t saturate_e4m3x4(uint32_t w) {
+  return w - ((((w & 0x7f7f7f7fu) + 0x01010101u) >> 7) & 0x01010101u);
 }
 
 template <int AUX>
@@ -141,6 +162,29 @@ __device__ __forceinline__ void store1(uint8_t v, __amdgpu_buffer_rsrc_t r, uint
 template <int SEL>
 __device__ __forceinline__ uint32_t cvt_e2m1x2(uint32_t w, float a, float b) {
   return __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, a, b, 1.0f, SEL);
+}
+
+// The same from two packed 16-bit values, each divided by `scale` (a power of
+// two given by its exponent field alone: 0 stands for 2^-127), and two e4m3fn
+// bytes in half HI of w likewise (overflow gives code 0x7f).  Every 16-bit
+// value at every scale byte 0-253 measured the same code as the binary32
+// product's conversion.
+template <int DT, int SEL>
+__device__ __forceinline__ uint32_t cvt_scaled_e2m1x2(uint32_t w, uint32_t y, float scale) {
+  if constexpr (DT == HPRMS_DTYPE_BF16)
+    return __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(w, __builtin_bit_cast(bf16x2, y), scale, SEL);
+  else
+    return __builtin_amdgcn_cvt_scalef32_pk_fp4_f16(w, __builtin_bit_cast(f16x2, y), scale, SEL);
+}
+
+typedef short s16x2 __attribute__((ext_vector_type(2)));
+template <int DT, bool HI>
+__device__ __forceinline__ uint32_t cvt_scaled_e4m3x2(uint32_t w, uint32_t y, float scale) {
+  const s16x2 o = __builtin_bit_cast(s16x2, w);
+  if constexpr (DT == HPRMS_DTYPE_BF16)
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(o, __builtin_bit_cast(bf16x2, y), scale, HI));
+  else
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_fp8_f16(o, __builtin_bit_cast(f16x2, y), scale, HI));
 }
 
 // ---- workgroup order ------------------------------------------------------------
@@ -196,6 +240,24 @@ __device__ __forceinline__ float group_sum(float v) {
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, false);
+}
+
+// max(m, |a|, |b|), NaN if any of them is (IEEE 754-2019 maximum; one gfx950
+// v_maximum3_f32).
+__device__ __forceinline__ float max_abs3(float m, float a, float b) {
+  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, __builtin_fabsf(a)), __builtin_fabsf(b));
+}
+
+// Lane LANE's value of each aligned group of 16 lanes, to all 16.
+template <int LANE>
+__device__ __forceinline__ float bcast16(float v) {
+  return dpp_f32<0x150 + LANE>(v);  // row_newbcast
+}
+
+// Lane LANE's value of each aligned quad, to all four.
+template <int LANE>
+__device__ __forceinline__ float bcast4(float v) {
+  return dpp_f32<LANE * 0x55>(v);  // quad_perm [LANE, LANE, LANE, LANE]
 }
 
 // Unsigned maximum over each aligned quad of lanes (every lane gets it).

@@ -148,9 +148,8 @@ struct FusedArgs {
 
 // Waves per SIMD the compiler must leave room for: the tail variant of the
 // 1024-lane shapes with up to 2 vectors per lane is held to 64 VGPRs, so two
-// workgroups share a CU as they do without the tail (the FP8 form needed 66:
-// held to 64 it runs 19-23% faster at 13K-16K).  At 3 vectors per lane the
-// same limit spills and measured 3-7% slower.  FLAGS bit 8 asks for 8 waves
+// workgroups share a CU as they do without the tail.  At 3 vectors per lane
+// the same limit spills and measured 3-7% slower.  FLAGS bit 8 asks for 8 waves
 // per SIMD (64 VGPRs) on any shape.
 template <int FLAGS, int BLOCK, int VPL>
 constexpr int kMinWavesPerEU = ((FLAGS & 256) != 0 || ((FLAGS & 64) != 0 && BLOCK == 1024 && VPL <= 2)) ? 8 : 1;
@@ -186,9 +185,9 @@ void fused_vec_kernel(const uint16_t* x_rows,  // input rows (MODE 0: also the o
   constexpr bool TAIL = (FLAGS & 64) != 0 && !BLOCKQ;              // shifted rows, head and tail vectors
   // rows off the 128-byte grid: each row's lane mapping rotated so that every
   // wave's 1 KiB access starts on a 512-byte boundary (`phases` bits 0-19)
-  // (not the FP8 and block-scaled outputs: the FP8 form's 1024 x 2 tail
-  // kernel, held to 64 VGPRs, would spill, and a block must stay one group
-  // of adjacent lanes)
+  // (not the FP8 and block-scaled outputs: their chunks are shorter than the
+  // rotation stream's, so they share lines with the next chunk either way, and
+  // a block must stay one group of adjacent lanes)
   constexpr bool ROT = (FLAGS & 32) != 0 && !BLOCKQ && MODE != 2;
   // residual loads issued first (not for the partial-sum form, where it measured 0.1-1.8% slower)
   constexpr bool RFIRST = (FLAGS & 128) != 0 && RES && MODE != 4;
@@ -482,8 +481,7 @@ void fused_vec_kernel(const uint16_t* x_rows,  // input rows (MODE 0: also the o
       const int64_t ss = opaque(a.mx_scale_stride);
       const uint32_t sbytes = (uint32_t)((int64_t)(nrows - 1) * ss + hidden / 32);
       xsrs = make_rsrc(sp + row0 * ss, sbytes);
-      // one lane of each quad writes its block's scale byte
-      xsoff = (lane & 3) == 0 ? (uint32_t)rib * (uint32_t)ss + (uint32_t)lane / 4u : kOOB;
+      xsoff = (uint32_t)rib * (uint32_t)ss + (uint32_t)lane / 4u;  // slot 0's block
     }
     if constexpr (GQ) {
       // float32 scales, one per 128 elements; scale (row, group) at byte
@@ -494,8 +492,7 @@ void fused_vec_kernel(const uint16_t* x_rows,  // input rows (MODE 0: also the o
       gs = (uint32_t)opaque(a.mx_group_stride);
       const uint32_t sbytes = (uint32_t)((int64_t)(nrows - 1) * ss + (int64_t)(hidden / 128 - 1) * gs + 4);
       xsrs = make_rsrc(sp + row0 * ss, sbytes);
-      // the first lane of each 16 writes its group's scale
-      xsoff = (lane & 15) == 0 ? (uint32_t)rib * (uint32_t)ss + (uint32_t)(lane / 16) * gs : kOOB;
+      xsoff = (uint32_t)rib * (uint32_t)ss + (uint32_t)(lane / 16) * gs;  // slot 0's group
     }
     if constexpr (MODE == 1) {
       // no residual: its (preloaded) arguments carry the output rows
@@ -710,80 +707,119 @@ void fused_vec_kernel(const uint16_t* x_rows,  // input rows (MODE 0: also the o
     // FLAGS bit 19 (bench library): the output phase at raised wave priority
     if constexpr ((FLAGS & 524288) != 0) __builtin_amdgcn_s_setprio(3);
 
+    // The quantised outputs.  Per lane and element these cost about as many
+    // vector instructions as the rest of the op, and with few rows per CU
+    // nothing hides them (a wave64 instruction takes four cycles), so: maxima
+    // are taken of the binary32 products (rounding is monotone, so the rounded
+    // maximum is the maximum of the rounded), one instruction per pair;
+    // per-block scales are computed once per lane group, by the lane whose
+    // number is the slot's, and broadcast by DPP; and nothing is clamped that
+    // cannot overflow (a value over its own group's maximum).
+    auto out_pair = [&](uint32_t s, uint32_t wp, float& m) {
+      const float p0 = (olo(s) * inv) * F::lo(wp), p1 = (ohi(s) * inv) * F::hi(wp);
+      m = max_abs3(m, p0, p1);
+      return F::pack(p0, p1);
+    };
+    auto held = [&](int k) { return k < VREG ? sv[k < VREG ? k : 0] : spill[(k - VREG) * BLOCK + tid]; };
     if constexpr (MX) {
       constexpr int EMAX = MODE == 5 ? 8 : 2;
+      // four slots at a time: lane j of a quad holds slot kb + j's block
+      each<(VPL + 3) / 4>([&](auto batch) {
+        constexpr int kb = batch * 4, KN = VPL - kb < 4 ? VPL - kb : 4;
+        float mine = 0.0f;
 #pragma unroll
-      for (int k = 0; k < VPL; ++k) {
-        const u32x4 s = k < VREG ? sv[k < VREG ? k : 0] : spill[(k - VREG) * BLOCK + tid];
-        u32x4 y;
-        uint32_t m2 = 0;
+        for (int j = 0; j < KN; ++j) {
+          const u32x4 s = held(kb + j);
+          float m = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          y[j] = F::pack((olo(s[j]) * inv) * F::lo(wv[k][j]), (ohi(s[j]) * inv) * F::hi(wv[k][j]));
-          const uint32_t mag = y[j] & 0x7fff7fffu;
-          m2 = __builtin_elementwise_max(m2, __builtin_elementwise_max(mag & 0xffffu, mag >> 16));
+          for (int i = 0; i < 4; ++i) xv[kb + j][i] = out_pair(s[i], wv[kb + j][i], m);
+          m = __uint_as_float(quad_max_u32(__float_as_uint(m)));
+          mine = (lane & 3) == j ? m : mine;
         }
         // the block maximum as binary32: its exponent field is floor(log2) + 127
         // (0 for zero and for bf16 subnormals, which clamp; 255 for NaN / inf)
-        const uint32_t e32 = __float_as_uint(F::one((uint16_t)quad_max_u32(m2))) >> 23;
-        int sexp = (int)e32 - 127 - EMAX;
-        if (e32 == 0 || sexp < -127) sexp = -127;
+        const uint32_t e32 = __float_as_uint(F::one(F::pack1(mine))) >> 23;
         const bool bad = e32 == 255u;
-        const float mul = bad ? 1.0f : __uint_as_float((uint32_t)(127 - sexp) << 23);
-        const bool ok = row_ok && vec_ok[k];
-        // a wave writes 16 consecutive scale bytes: default cache policy, so
-        // that L2 merges the pieces of a line before it goes to memory
-        store1<0>((uint8_t)(bad ? 0xFFu : (uint32_t)(sexp + 127)), xsrs,
-                  ok && xsoff != kOOB ? xsoff + (uint32_t)(k * (LPR / 4)) : kOOB);
-        if constexpr (MODE == 5) {
-          u32x2 q;
+        // the scale byte s + 127, at least 0; a bad block's elements are unscaled
+        const uint32_t sb = e32 > (uint32_t)EMAX ? e32 - EMAX : 0u;
+        const float fac = __uint_as_float((bad ? 127u : sb) << 23);
+        const int slot = kb + (lane & 3);
+        // a wave writes 16 consecutive scale bytes per slot: default cache
+        // policy, so that L2 merges the pieces of a line before it goes to memory
+        store1<0>((uint8_t)(bad ? 0xFFu : sb), xsrs,
+                  row_ok && slot < VPL && slot * LPR + lane < nvec ? xsoff + (uint32_t)(slot * (LPR / 4)) : kOOB);
+        const bool any_bad = MODE == 5 && __builtin_amdgcn_ballot_w64(bad) != 0;
+        each<KN>([&](auto j) {
+          constexpr int k = kb + j;
+          const u32x4 y = xv[k];
+          const float f = bcast4<j>(fac);
+          const bool ok = row_ok && vec_ok[k];
+          if constexpr (MODE == 5) {
+            u32x2 q;
+            if (any_bad) {
+              // some block of this wave holds NaN or infinity, or is unscaled
+              // for it: NaN must stay, everything else saturate
+              const float mul = __uint_as_float((254u << 23) - __float_as_uint(f));
 #pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const uint32_t y0 = y[2 * h], y1 = y[2 * h + 1];
-            q[h] = pack_e4m3x4(clamp_e4m3(F::lo(y0) * mul), clamp_e4m3(F::hi(y0) * mul),
-                               clamp_e4m3(F::lo(y1) * mul), clamp_e4m3(F::hi(y1) * mul));
+              for (int h = 0; h < 2; ++h) {
+                const uint32_t y0 = y[2 * h], y1 = y[2 * h + 1];
+                q[h] = pack_e4m3x4(clamp_e4m3(F::lo(y0) * mul), clamp_e4m3(F::hi(y0) * mul),
+                                   clamp_e4m3(F::lo(y1) * mul), clamp_e4m3(F::hi(y1) * mul));
+              }
+            } else {
+              // the block's values are below 2^9 once scaled: those past 464
+              // convert to the overflow code
+#pragma unroll
+              for (int h = 0; h < 2; ++h)
+                q[h] = saturate_e4m3x4(cvt_scaled_e4m3x2<DT, true>(cvt_scaled_e4m3x2<DT, false>(0u, y[2 * h], f),
+                                                                   y[2 * h + 1], f));
+            }
+            store8<OSAUX>(q, ors, ok ? ooff + k * (LPR * 8u) : kOOB);
+          } else {
+            uint32_t q = 0;
+            q = cvt_scaled_e2m1x2<DT, 0>(q, y[0], f);
+            q = cvt_scaled_e2m1x2<DT, 1>(q, y[1], f);
+            q = cvt_scaled_e2m1x2<DT, 2>(q, y[2], f);
+            q = cvt_scaled_e2m1x2<DT, 3>(q, y[3], f);
+            store4<OSAUX>(q, ors, ok ? ooff + k * (LPR * 4u) : kOOB);
           }
-          store8<OSAUX>(q, ors, ok ? ooff + k * (LPR * 8u) : kOOB);
-        } else {
-          uint32_t q = 0;
-          q = cvt_e2m1x2<0>(q, F::lo(y[0]) * mul, F::hi(y[0]) * mul);
-          q = cvt_e2m1x2<1>(q, F::lo(y[1]) * mul, F::hi(y[1]) * mul);
-          q = cvt_e2m1x2<2>(q, F::lo(y[2]) * mul, F::hi(y[2]) * mul);
-          q = cvt_e2m1x2<3>(q, F::lo(y[3]) * mul, F::hi(y[3]) * mul);
-          store4<OSAUX>(q, ors, ok ? ooff + k * (LPR * 4u) : kOOB);
-        }
-      }
+        });
+      });
     } else if constexpr (GQ) {
+      // lane j of the 16 lanes that share a group at each slot holds slot j's
+      // maximum, so the two divisions and the store are done once, not per slot
+      static_assert(VPL <= 16, "a lane per slot");
+      float mine = 0.0f;
 #pragma unroll
       for (int k = 0; k < VPL; ++k) {
-        const u32x4 s = k < VREG ? sv[k < VREG ? k : 0] : spill[(k - VREG) * BLOCK + tid];
-        u32x4 y;
-        uint32_t m2 = 0;
+        const u32x4 s = held(k);
+        float m = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          y[j] = F::pack((olo(s[j]) * inv) * F::lo(wv[k][j]), (ohi(s[j]) * inv) * F::hi(wv[k][j]));
-          const uint32_t mag = y[j] & 0x7fff7fffu;
-          m2 = __builtin_elementwise_max(m2, __builtin_elementwise_max(mag & 0xffffu, mag >> 16));
-        }
-        // the group's maximum magnitude: the 16 lanes of a DPP row hold its
-        // 16 vectors (sign-magnitude patterns order like their values, NaN
-        // above inf)
-        const float amax = F::one((uint16_t)group_max_u32<16>(m2));
-        float sc = amax / 448.0f;
-        if (sc < 1.17549435e-38f) sc = 1.17549435e-38f;  // FLT_MIN; NaN stays NaN
-        const float isc = 1.0f / sc;
+        for (int i = 0; i < 4; ++i) xv[k][i] = out_pair(s[i], wv[k][i], m);
+        m = __uint_as_float(group_max_u32<16>(__float_as_uint(m)));
+        mine = (lane & 15) == k ? m : mine;
+      }
+      const float amax = F::one(F::pack1(mine));
+      float sc = amax / 448.0f;
+      if (sc < 1.17549435e-38f) sc = 1.17549435e-38f;  // FLT_MIN; NaN stays NaN
+      const float isc = 1.0f / sc;
+      const int slot = lane & 15;
+      // default cache policy, so that L2 merges a row's scales into lines
+      store4<0>(__float_as_uint(sc), xsrs,
+                row_ok && slot < VPL && slot * LPR + lane < nvec ? xsoff + (uint32_t)(slot * (LPR / 16)) * gs : kOOB);
+      each<VPL>([&](auto j) {
+        constexpr int k = j;
+        const u32x4 y = xv[k];
+        const float f = bcast16<k>(isc);
         const bool ok = row_ok && vec_ok[k];
-        // default cache policy, so that L2 merges a row's scales into lines
-        store4<0>(__float_as_uint(sc), xsrs, ok && xsoff != kOOB ? xsoff + (uint32_t)(k * (LPR / 16)) * gs : kOOB);
         u32x2 q;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const uint32_t y0 = y[2 * h], y1 = y[2 * h + 1];
-          q[h] = pack_e4m3x4(clamp_e4m3(F::lo(y0) * isc), clamp_e4m3(F::hi(y0) * isc),
-                             clamp_e4m3(F::lo(y1) * isc), clamp_e4m3(F::hi(y1) * isc));
+          q[h] = pack_e4m3x4(F::lo(y0) * f, F::hi(y0) * f, F::lo(y1) * f, F::hi(y1) * f);
         }
         store8<OSAUX>(q, ors, ok ? ooff + k * (LPR * 8u) : kOOB);
-      }
+      });
     } else if constexpr (MODE != 2) {
 #pragma unroll
       for (int k = 0; k < VPL; ++k) {
@@ -803,37 +839,20 @@ void fused_vec_kernel(const uint16_t* x_rows,  // input rows (MODE 0: also the o
         store16<OSAUX>(o, ors, eooff);
       }
     } else {
-      // y in 16-bit form, kept in the registers x came in; the row maximum of
-      // |y| over the valid vectors, as packed 16-bit magnitudes
-      uint32_t m2 = 0;
+      // y in 16-bit form, kept in the registers x came in, and the row maximum
+      // of |y|.  Slots past the row hold zeros and zero weights: they add a 0,
+      // or a NaN (0 times an infinite or NaN inv) that the row's own elements
+      // give too.  The edge vector's repeated elements are harmless.
+      float m = 0.0f;
 #pragma unroll
       for (int k = 0; k < VPL; ++k) {
-        const u32x4 s = k < VREG ? sv[k < VREG ? k : 0] : spill[(k - VREG) * BLOCK + tid];
+        const u32x4 s = held(k);
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          xv[k][j] = F::pack((olo(s[j]) * inv) * F::lo(wv[k][j]), (ohi(s[j]) * inv) * F::hi(wv[k][j]));
-        if (row_ok && vec_ok[k]) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const uint32_t mag = xv[k][j] & 0x7fff7fffu;
-            const uint32_t lo = mag & 0xffffu, hi = mag >> 16;
-            m2 = __builtin_elementwise_max(m2, __builtin_elementwise_max(lo, hi));
-          }
-        }
+        for (int j = 0; j < 4; ++j) xv[k][j] = out_pair(s[j], wv[k][j], m);
       }
       if constexpr (TAIL) {
-        // the edge vector's elements outside [elo, ehi) repeat ones already
-        // counted: harmless for a maximum
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          txv[j] = F::pack((olo(tsv[j]) * inv) * F::lo(twv[j]), (ohi(tsv[j]) * inv) * F::hi(twv[j]));
-        if (eok) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const uint32_t mag = txv[j] & 0x7fff7fffu;
-            m2 = __builtin_elementwise_max(m2, __builtin_elementwise_max(mag & 0xffffu, mag >> 16));
-          }
-        }
+        for (int j = 0; j < 4; ++j) txv[j] = out_pair(tsv[j], twv[j], m);
       }
       float isc;
       if (has_given) {
@@ -842,7 +861,7 @@ void fused_vec_kernel(const uint16_t* x_rows,  // input rows (MODE 0: also the o
         // part of it)
         isc = 1.0f / given_scale;
       } else {
-        uint32_t mx = group_max_u32<GW>(m2);
+        uint32_t mx = group_max_u32<GW>(__float_as_uint(m));
         if constexpr (WPR > 1) {
           if ((tid & 63) == 0) red[buf][wave] = __builtin_bit_cast(float, mx);
           __syncthreads();
@@ -852,35 +871,38 @@ void fused_vec_kernel(const uint16_t* x_rows,  // input rows (MODE 0: also the o
             mx = __builtin_elementwise_max(mx, __builtin_bit_cast(uint32_t, red[buf][w0 + j]));
           buf ^= 1;
         }
-        float amax = F::one((uint16_t)mx);
+        float amax = F::one(F::pack1(__uint_as_float(mx)));
         if (amax > ubound) amax = ubound;  // the caller's bound (a NaN maximum stays NaN)
         float sc = amax / 448.0f;
         if (sc < 1.17549435e-38f) sc = 1.17549435e-38f;  // FLT_MIN; NaN stays NaN
         isc = 1.0f / sc;
         if (row_ok && lane == 0) opaque(a.scale)[row0 + rib] = sc;
       }
+      // only a given scale or a bound (NaN: none) lets a value pass 448: a
+      // row's own maximum scales to 448 within two roundings, and the
+      // conversion rounds up to 464 down to it
+      auto quantise = [&](auto clamped) {
+        auto one8 = [&](const u32x4& y) {
+          auto c = [](float v) { if constexpr (decltype(clamped)::value) return clamp_e4m3(v); else return v; };
+          u32x2 q;
 #pragma unroll
-      for (int k = 0; k < VPL; ++k) {
-        u32x2 q;
+          for (int h = 0; h < 2; ++h) {
+            const uint32_t y0 = y[2 * h], y1 = y[2 * h + 1];
+            q[h] = pack_e4m3x4(c(F::lo(y0) * isc), c(F::hi(y0) * isc), c(F::lo(y1) * isc), c(F::hi(y1) * isc));
+          }
+          return q;
+        };
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const uint32_t y0 = xv[k][2 * h], y1 = xv[k][2 * h + 1];
-          q[h] = pack_e4m3x4(clamp_e4m3(F::lo(y0) * isc), clamp_e4m3(F::hi(y0) * isc),
-                             clamp_e4m3(F::lo(y1) * isc), clamp_e4m3(F::hi(y1) * isc));
+        for (int k = 0; k < VPL; ++k) {
+          const bool ok = row_ok && vec_ok[k];
+          store8<OSAUX>(one8(xv[k]), ors, ok ? ooff + k * (LPR * 8u) + (k == 0 ? wrap * 8u : 0u) : kOOB);
         }
-        const bool ok = row_ok && vec_ok[k];
-        store8<OSAUX>(q, ors, ok ? ooff + k * (LPR * 8u) + (k == 0 ? wrap * 8u : 0u) : kOOB);
-      }
-      if constexpr (TAIL) {
-        u32x2 q;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const uint32_t y0 = txv[2 * h], y1 = txv[2 * h + 1];
-          q[h] = pack_e4m3x4(clamp_e4m3(F::lo(y0) * isc), clamp_e4m3(F::hi(y0) * isc),
-                             clamp_e4m3(F::lo(y1) * isc), clamp_e4m3(F::hi(y1) * isc));
-        }
-        store8<OSAUX>(q, ors, eooff);
-      }
+        if constexpr (TAIL) store8<OSAUX>(one8(txv), ors, eooff);
+      };
+      if (has_given || ubound == ubound)
+        quantise(std::true_type{});
+      else
+        quantise(std::false_type{});
     }
     if constexpr ((FLAGS & 524288) != 0) __builtin_amdgcn_s_setprio(0);
     g += grid;

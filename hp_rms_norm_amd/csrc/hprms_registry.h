@@ -119,7 +119,7 @@ struct FusedEntry {
 // rows, for bench.py --ab-runs
 #define HPRMS_QUANT_RUNS_AB(X, DT)                                                                 \
   X(DT, 2, 256, 2, 0, 256, 7 | 327680) X(DT, 5, 256, 2, 0, 256, 7 | 327680)                       \
-  X(DT, 6, 256, 2, 0, 256, 7 | 327680) X(DT, 7, 1024, 2, 0, 1024, 31 | 327680)                    \
+  X(DT, 6, 256, 2, 0, 256, 7 | 327680) X(DT, 7, 256, 8, 0, 256, 7 | 327680)                       \
   X(DT, 7, 1024, 4, 0, 1024, 159 | 327680)                                                        \
   X(DT, 1, 64, 8, 0, 256, 3 | 327680) X(DT, 1, 64, 8, 0, 256, 3 | 393216)                         \
   X(DT, 1, 512, 2, 0, 512, 31 | 327680) X(DT, 1, 512, 2, 0, 512, 31 | 393216)                     \
@@ -144,10 +144,12 @@ struct FusedEntry {
 
 // the FP8 output (mode 2) and the OCP MX outputs (modes 5 and 6)
 #define HPRMS_QUANT_SHAPES(X, DT, MODE)                                                           \
-  HPRMS_COMMON_SHAPES(X, DT, MODE) X(DT, MODE, 1024, 3, 0, 1024, 159)                              \
-  X(DT, MODE, 128, 3, 0, 256, 7) X(DT, MODE, 256, 3, 0, 256, 7) X(DT, MODE, 1024, 2, 0, 1024, 31)
+  HPRMS_COMMON_SHAPES(X, DT, MODE)                                                               \
+  X(DT, MODE, 128, 3, 0, 256, 7) X(DT, MODE, 256, 3, 0, 256, 7)                                   \
+  X(DT, MODE, 512, 5, 0, 512, 135) X(DT, MODE, 512, 6, 0, 512, 135)
 #define HPRMS_MODE2_SHAPES(X, DT, MODE) HPRMS_QUANT_SHAPES(X, DT, MODE) X(DT, MODE, 512, 8, 4, 512, 159)
-#define HPRMS_MX_SHAPES(X, DT, MODE) HPRMS_QUANT_SHAPES(X, DT, MODE) X(DT, MODE, 1024, 4, 0, 1024, 159)
+#define HPRMS_MX_SHAPES(X, DT, MODE) \
+  HPRMS_QUANT_SHAPES(X, DT, MODE) X(DT, MODE, 256, 8, 0, 256, 7) X(DT, MODE, 1024, 4, 0, 1024, 159)
 
 // Every mode's lists for one registry: the kernels for rows on the 128-byte
 // grid (ENTRY = HPRMS_FUSED_ENTRY), and for rows off it (the unaligned and
@@ -210,7 +212,8 @@ struct FusedEntry {
   X(DT, MODE, 128, 4, 0, 256, 131) X(DT, MODE, 256, 4, 0, 256, 3) X(DT, MODE, 256, 3, 0, 256, 7)  \
   X(DT, MODE, 512, 8, 4, 512, 159) X(DT, MODE, 64, 8, 0, 256, 3) X(DT, MODE, 512, 2, 0, 512, 31)  \
   X(DT, MODE, 512, 4, 0, 512, 31) X(DT, MODE, 512, 8, 0, 512, 7) X(DT, MODE, 1024, 2, 0, 1024, 31) \
-  X(DT, MODE, 1024, 3, 0, 1024, 159)
+  X(DT, MODE, 1024, 3, 0, 1024, 159) X(DT, MODE, 256, 8, 0, 256, 7) X(DT, MODE, 512, 5, 0, 512, 135) \
+  X(DT, MODE, 512, 6, 0, 512, 135)
 
 // The shapes below are built only into the bench library libhprms_bench.so
 // (hprms.hip compiled with HPRMS_BENCH_BUILD), never into libhprms.so: no
