@@ -446,19 +446,23 @@ void table_config(int64_t rows, int64_t hidden, int mode, bool grid, int cus, hp
 // bits are the same.
 // The quantised outputs (modes 2, 5, 6, 7) at 16 KiB rows with their table
 // kernel (512 x 2), runs of 32: 0.3-1.1% faster at 4096 rows (seven
-// interleaved trials), and 5.7% for mode 7 with column-major scales.  Those
-// scales are 4-byte stores, 32 rows to a 128-byte line; with one row per
-// workgroup the 32 rows of a line otherwise go to all 8 XCDs, and each XCD's
-// L2 writes its part of the line back on its own.  Mode 7 with column-major
-// scales also takes runs of 32 at 8 KiB rows (256 x 2): 2.2-3.5% faster;
-// there modes 2, 5 and 6 were within 0.4% either way, and mode 7 with rows
-// of scales from 1.1% faster to 0.5% slower over two boxes, so left out.  At
-// 32 and 64 KiB rows (1024 lanes, one row per workgroup) runs of 8-64 were
-// 3-13% slower in mode 7.
+// interleaved trials).  Mode 7's column-major scales are 4-byte stores, 32
+// rows to a 128-byte line; with one row per workgroup the 32 rows of a line
+// otherwise go to all 8 XCDs, and each XCD's L2 writes its part of the line
+// back on its own.  That cost does not depend on the pitch, so with such
+// scales mode 7 takes the same runs at every width of 256 x 2 (3K < H <= 4K)
+// and 512 x 2 (5K < H <= 8K) from 1024 rows, four rounds of the XCDs' runs
+// (bf16, cold, interleaved trials; 1024 / 2048 / 4096 / 8192 rows: 7168
+// columns 2.2 / 2.0 / 4.0 / 2.1% faster, 36.9 -> 35.5 us at 4096; 6144 2.5 /
+// 2.3 / 3.7 / 3.0%, 4096 2.3 / 2.4 / 2.8 / 2.6%, 8192 2.3 / 3.1 / 5.6 / 2.2%;
+// at 512 rows -1% to +3.7%: left out).  With rows of scales mode 7 ranged from
+// 1.1% faster to 0.6% slower, and at 8 KiB rows modes 2, 5 and 6 were within
+// 0.4% either way, so left out.  At 32 and 64 KiB rows (1024 lanes, one row
+// per workgroup) runs of 8-64 were 3-13% slower in mode 7.
 struct RunsRow {
   unsigned modes;       // bit m: mode m
   bool scale_columns;   // mode 7 with column-major scales only
-  int64_t pitch_bytes;
+  int64_t pitch_bytes;  // 0: any
   int lpr, vpl, block, flags, v;
   int64_t min_rows;  // on 256 CUs
 };
@@ -466,7 +470,8 @@ constexpr unsigned kQuantModes = 1u << 2 | 1u << 5 | 1u << 6 | 1u << 7;
 constexpr RunsRow kRuns[] = {{1u, false, 8192, 256, 2, 256, 131, 5, 4096},
                              {1u, false, 16384, 512, 2, 512, 7, 6, 2048},
                              {kQuantModes, false, 16384, 512, 2, 512, 7, 5, 4096},
-                             {1u << 7, true, 8192, 256, 2, 256, 7, 5, 4096}};
+                             {1u << 7, true, 0, 256, 2, 256, 7, 5, 1024},
+                             {1u << 7, true, 0, 512, 2, 512, 7, 5, 1024}};
 
 // flags bits 16-18 for configuration c of mode `mode` on rows `pitch_bytes`
 // apart in both input streams, on the 128-byte grid (scale_columns: mode 7's
@@ -475,8 +480,9 @@ int xcd_runs_flags(int mode, int64_t rows, int64_t pitch_bytes, int cus, const h
                    bool scale_columns) {
   if (c.tier != 1 || c.lds_vec_per_lane != 0) return 0;
   for (const RunsRow& r : kRuns)
-    if (((r.modes >> mode) & 1u) && (!r.scale_columns || scale_columns) && r.pitch_bytes == pitch_bytes &&
-        r.lpr == c.lanes_per_row && r.vpl == c.vec_per_lane && r.block == c.block_threads && r.flags == c.flags &&
+    if (((r.modes >> mode) & 1u) && (!r.scale_columns || scale_columns) &&
+        (r.pitch_bytes == 0 || r.pitch_bytes == pitch_bytes) && r.lpr == c.lanes_per_row &&
+        r.vpl == c.vec_per_lane && r.block == c.block_threads && r.flags == c.flags &&
         rows_at_ref(rows, cus) >= r.min_rows)
       return r.v << 16;
   return 0;

@@ -107,8 +107,8 @@ struct FusedEntry {
 // the in-place op's rows with their row groups in runs per XCD (hprms.hip, kRuns)
 #define HPRMS_RUNS_ROWS(X, DT, MODE) X(DT, MODE, 256, 2, 0, 256, 131 | 327680) X(DT, MODE, 512, 2, 0, 512, 7 | 393216)
 // the quantised outputs' rows with runs of 32 row groups per XCD (hprms.hip,
-// kRuns; aligned registry only): 16 KiB rows in modes 2, 5, 6, 7, and 8 KiB
-// rows in mode 7 (column-major scales)
+// kRuns; aligned registry only): 16 KiB rows in modes 2, 5, 6, 7, and mode 7
+// with column-major scales in 256 x 2 and 512 x 2
 #define HPRMS_QUANT_RUNS(X, DT)                                                                    \
   X(DT, 2, 512, 2, 0, 512, 7 | 327680) X(DT, 5, 512, 2, 0, 512, 7 | 327680)                       \
   X(DT, 6, 512, 2, 0, 512, 7 | 327680) X(DT, 7, 512, 2, 0, 512, 7 | 327680)                       \

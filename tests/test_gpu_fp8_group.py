@@ -213,6 +213,15 @@ def test_fp8_group_column_major_scales_through_the_abi(ops, rows, hidden, pad):
     assert_fp8_from_y_within_one_ulp(q_bits(q), oy, np.repeat(np.float32(1.0) / scales, 128, axis=1), torch.bfloat16)
 
 
+@pytest.mark.parametrize("rows,hidden,pad", [(1023, 7168, 0), (1024, 3200, 0), (1024, 8192, 1), (1281, 5248, 3),
+                                             (1536, 4096, 0)])
+def test_fp8_group_column_major_runs_edges(ops, rows, hidden, pad):
+    """Around the first row count of the runs per XCD, and row counts that end
+    inside a run's block of 256 row groups: each row written once, and the
+    same bits as with rows of scales."""
+    test_fp8_group_column_major_scales_through_the_abi(ops, rows, hidden, pad)
+
+
 def test_fp8_group_column_major_scales_through_the_torch_op(ops):
     """The allocating form with column-major scales, 16-byte aligned columns
     (tokens rounded up to a multiple of 4), on a [batch, seq, H] input; and the
