@@ -227,20 +227,33 @@ bool latency_config(int64_t rows, int64_t nvec, int mode, hprms_config* c) {
 // 4096.  Past 24K the LDS tier (per row) and 1024 x 4 (per block) stay, 2-5%
 // ahead of 512 x 8 in registers.  256 x 8 against 512 x 4 at 16384: MXFP4
 // 2-4% and FP8 per 128 elements 2% faster, per-row FP8 the same.
-bool quant_config(int64_t nvec, int mode, hprms_config* c) {
+// 256 x 2 and 512 x 2 load the weight with the row (flags 3) in the per-row
+// FP8 and MX forms: their output phase is long enough that a weight load
+// issued after the residual's stores is waited for with nothing else to do.
+// Cold, interleaved trials, bf16, H = 3584-8192 at 1024 / 2048 / 4096 / 8192
+// rows: per-row FP8 2.0-4.0 / 1.4-3.6 / 0.2-1.7 / up to 1.3% faster (2048 x
+// 8192: 21.8 -> 21.5 us), MXFP8 1.4-5.6 / 1.2-4.9 / 0-2.1 / within 0.9%,
+// MXFP4 1.3-7.2 / 2.3-4.0 / 0.5-1.4 / within 0.6%.  Per-row FP8 keeps the late
+// weight off the 128-byte grid (`grid`: its tail variant holds an edge vector
+// too); so do 256 x 3 (early: MX 4% faster at 1024 rows, 1.5% slower at 8192,
+// FP8 3.5% faster to 1.3% slower) and FP8 per 128 elements.
+bool quant_config(int64_t nvec, int mode, bool grid, hprms_config* c) {
   struct Row { unsigned modes; int64_t min_nvec, max_nvec; int lpr, vpl, ldsv, block, flags; };
-  constexpr unsigned all = ~0u, row = 1u << 2, blocks = ~row;
-  static const Row quant[] = {{all, 129, 256, 128, 2, 0, 128, 3},
-                              {all, 385, 512, 256, 2, 0, 256, 7},
-                              {all, 513, 640, 256, 3, 0, 256, 7},
-                              {all, 641, 1024, 512, 2, 0, 512, 7},
-                              {row, 1537, 2048, 512, 4, 0, 512, 7},
-                              {blocks, 1537, 1792, 512, 4, 0, 512, 7},
-                              {blocks, 1793, 2048, 256, 8, 0, 256, 7},
-                              {all, 2049, 2560, 512, 5, 0, 512, 135},
-                              {all, 2561, 3072, 512, 6, 0, 512, 135},
-                              {row, 3073, 4096, 512, 8, 4, 512, 159},
-                              {blocks, 3073, 4096, 1024, 4, 0, 1024, 159}};
+  constexpr unsigned all = ~0u, row = 1u << 2, blocks = ~row, mx = 1u << 5 | 1u << 6;
+  const unsigned early = grid ? row | mx : mx;
+  const Row quant[] = {{all, 129, 256, 128, 2, 0, 128, 3},
+                       {early, 385, 512, 256, 2, 0, 256, 3},
+                       {all, 385, 512, 256, 2, 0, 256, 7},
+                       {all, 513, 640, 256, 3, 0, 256, 7},
+                       {early, 641, 1024, 512, 2, 0, 512, 3},
+                       {all, 641, 1024, 512, 2, 0, 512, 7},
+                       {row, 1537, 2048, 512, 4, 0, 512, 7},
+                       {blocks, 1537, 1792, 512, 4, 0, 512, 7},
+                       {blocks, 1793, 2048, 256, 8, 0, 256, 7},
+                       {all, 2049, 2560, 512, 5, 0, 512, 135},
+                       {all, 2561, 3072, 512, 6, 0, 512, 135},
+                       {row, 3073, 4096, 512, 8, 4, 512, 159},
+                       {blocks, 3073, 4096, 1024, 4, 0, 1024, 159}};
   for (const Row& r : quant) {
     if (((r.modes >> mode) & 1u) && nvec >= r.min_nvec && nvec <= r.max_nvec) {
       *c = hprms_config{r.ldsv > 0 ? 2 : 1, r.lpr, r.vpl, r.ldsv, r.block, 0, r.flags};
@@ -392,7 +405,7 @@ void table_config(int64_t rows, int64_t hidden, int mode, bool grid, int cus, hp
   if (mode == 0 && grid && inplace_config(nvec, c)) return;
   if (mode == 1 && plain_config(nvec, c)) return;
   if (mode == 4 && reduce_config(nvec, c)) return;
-  if ((mode == 2 || mode >= 5) && quant_config(nvec, mode, c)) return;
+  if ((mode == 2 || mode >= 5) && quant_config(nvec, mode, grid, c)) return;
   *c = hprms_config{1, 0, 0, 0, 0, 0, 3};
   // flags: 3 = non-temporal row loads and stores, +4 = weight loaded late,
   // +24 = sc1 on loads and stores, +128 = residual loads before input loads
@@ -445,7 +458,7 @@ void table_config(int64_t rows, int64_t hidden, int mode, bool grid, int cus, hp
 // the row count.  The order only changes which workgroup takes a row, so the
 // bits are the same.
 // The quantised outputs (modes 2, 5, 6, 7) at 16 KiB rows with their table
-// kernel (512 x 2), runs of 32: 0.3-1.1% faster at 4096 rows (seven
+// kernel (512 x 2), runs of 32: 0.3-1.5% faster at 4096 rows (seven
 // interleaved trials).  Mode 7's column-major scales are 4-byte stores, 32
 // rows to a 128-byte line; with one row per workgroup the 32 rows of a line
 // otherwise go to all 8 XCDs, and each XCD's L2 writes its part of the line
@@ -466,10 +479,11 @@ struct RunsRow {
   int lpr, vpl, block, flags, v;
   int64_t min_rows;  // on 256 CUs
 };
-constexpr unsigned kQuantModes = 1u << 2 | 1u << 5 | 1u << 6 | 1u << 7;
+constexpr unsigned kRowMxModes = 1u << 2 | 1u << 5 | 1u << 6;
 constexpr RunsRow kRuns[] = {{1u, false, 8192, 256, 2, 256, 131, 5, 4096},
                              {1u, false, 16384, 512, 2, 512, 7, 6, 2048},
-                             {kQuantModes, false, 16384, 512, 2, 512, 7, 5, 4096},
+                             {kRowMxModes, false, 16384, 512, 2, 512, 3, 5, 4096},
+                             {1u << 7, false, 16384, 512, 2, 512, 7, 5, 4096},
                              {1u << 7, true, 0, 256, 2, 256, 7, 5, 1024},
                              {1u << 7, true, 0, 512, 2, 512, 7, 5, 1024}};
 

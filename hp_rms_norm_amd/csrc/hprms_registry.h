@@ -110,16 +110,19 @@ struct FusedEntry {
 // kRuns; aligned registry only): 16 KiB rows in modes 2, 5, 6, 7, and mode 7
 // with column-major scales in 256 x 2 and 512 x 2
 #define HPRMS_QUANT_RUNS(X, DT)                                                                    \
-  X(DT, 2, 512, 2, 0, 512, 7 | 327680) X(DT, 5, 512, 2, 0, 512, 7 | 327680)                       \
-  X(DT, 6, 512, 2, 0, 512, 7 | 327680) X(DT, 7, 512, 2, 0, 512, 7 | 327680)                       \
+  X(DT, 2, 512, 2, 0, 512, 3 | 327680) X(DT, 5, 512, 2, 0, 512, 3 | 327680)                       \
+  X(DT, 6, 512, 2, 0, 512, 3 | 327680) X(DT, 7, 512, 2, 0, 512, 7 | 327680)                       \
   X(DT, 7, 256, 2, 0, 256, 7 | 327680)
 // bench library: the same runs where the table leaves them out (modes 2, 5, 6
-// at 8 KiB rows; mode 7 at 32 and 64 KiB rows), and runs of 32 and 64 for the
+// at 8 KiB rows, and with the late weight at 16 KiB; mode 7 at 32 and 64 KiB
+// rows), and runs of 32 and 64 for the
 // plain RMSNorm (mode 1) and the op out of place (mode 3) at 8 and 16 KiB
 // rows, for bench.py --ab-runs
 #define HPRMS_QUANT_RUNS_AB(X, DT)                                                                 \
-  X(DT, 2, 256, 2, 0, 256, 7 | 327680) X(DT, 5, 256, 2, 0, 256, 7 | 327680)                       \
-  X(DT, 6, 256, 2, 0, 256, 7 | 327680) X(DT, 7, 256, 8, 0, 256, 7 | 327680)                       \
+  X(DT, 2, 256, 2, 0, 256, 3 | 327680) X(DT, 5, 256, 2, 0, 256, 3 | 327680)                       \
+  X(DT, 2, 512, 2, 0, 512, 7 | 327680) X(DT, 5, 512, 2, 0, 512, 7 | 327680)                       \
+  X(DT, 6, 512, 2, 0, 512, 7 | 327680)                                                           \
+  X(DT, 6, 256, 2, 0, 256, 3 | 327680) X(DT, 7, 256, 8, 0, 256, 7 | 327680)                       \
   X(DT, 7, 1024, 4, 0, 1024, 159 | 327680)                                                        \
   X(DT, 1, 64, 8, 0, 256, 3 | 327680) X(DT, 1, 64, 8, 0, 256, 3 | 393216)                         \
   X(DT, 1, 512, 2, 0, 512, 31 | 327680) X(DT, 1, 512, 2, 0, 512, 31 | 393216)                     \
@@ -147,9 +150,13 @@ struct FusedEntry {
   HPRMS_COMMON_SHAPES(X, DT, MODE)                                                               \
   X(DT, MODE, 128, 3, 0, 256, 7) X(DT, MODE, 256, 3, 0, 256, 7)                                   \
   X(DT, MODE, 512, 5, 0, 512, 135) X(DT, MODE, 512, 6, 0, 512, 135)
+// the MX rows, and the per-row FP8 rows on the 128-byte grid, that load the
+// weight with the row
+#define HPRMS_QUANT_EARLY(X, DT, MODE) X(DT, MODE, 256, 2, 0, 256, 3) X(DT, MODE, 512, 2, 0, 512, 3)
 #define HPRMS_MODE2_SHAPES(X, DT, MODE) HPRMS_QUANT_SHAPES(X, DT, MODE) X(DT, MODE, 512, 8, 4, 512, 159)
-#define HPRMS_MX_SHAPES(X, DT, MODE) \
+#define HPRMS_BLOCKQ_SHAPES(X, DT, MODE) \
   HPRMS_QUANT_SHAPES(X, DT, MODE) X(DT, MODE, 256, 8, 0, 256, 7) X(DT, MODE, 1024, 4, 0, 1024, 159)
+#define HPRMS_MX_SHAPES(X, DT, MODE) HPRMS_BLOCKQ_SHAPES(X, DT, MODE) HPRMS_QUANT_EARLY(X, DT, MODE)
 
 // Every mode's lists for one registry: the kernels for rows on the 128-byte
 // grid (ENTRY = HPRMS_FUSED_ENTRY), and for rows off it (the unaligned and
@@ -159,7 +166,7 @@ struct FusedEntry {
   HPRMS_MODE4_SHAPES(ENTRY, DT, 4)
 #define HPRMS_ALL_MODES(ENTRY, DT) \
   HPRMS_MODE0_SHAPES(ENTRY, DT, 0) HPRMS_MODES_1_TO_4(ENTRY, DT) HPRMS_WAVE_ROWS(ENTRY, DT, 3) \
-  HPRMS_WAVE_ROWS(ENTRY, DT, 1) \
+  HPRMS_WAVE_ROWS(ENTRY, DT, 1) HPRMS_QUANT_EARLY(ENTRY, DT, 2) \
   HPRMS_PAIR_ROWS(ENTRY, DT, 3)
 #define HPRMS_ALL_MODES_OFFGRID(ENTRY, DT) HPRMS_MODE0_OFFGRID_SHAPES(ENTRY, DT, 0) HPRMS_MODES_1_TO_4(ENTRY, DT)
 #define HPRMS_ALL_MODES_TAIL(ENTRY, DT)                                                           \
@@ -168,9 +175,9 @@ struct FusedEntry {
   HPRMS_FUSED_TAIL_SHAPES(ENTRY, DT, 3) ENTRY(DT, 3, 128, 4, 0, 256, 131) HPRMS_WIDE_ROWS(ENTRY, DT, 3) \
   HPRMS_MODE4_TAIL_SHAPES(ENTRY, DT, 4) ENTRY(DT, 4, 128, 4, 0, 256, 131) ENTRY(DT, 4, 256, 4, 0, 256, 3)
 // the block-scaled outputs: MX (modes 5, 6) and FP8 with a scale per 128
-// elements (mode 7), with the same shapes
+// elements (mode 7)
 #define HPRMS_MX_MODES(ENTRY, DT) \
-  HPRMS_MX_SHAPES(ENTRY, DT, 5) HPRMS_MX_SHAPES(ENTRY, DT, 6) HPRMS_MX_SHAPES(ENTRY, DT, 7)
+  HPRMS_MX_SHAPES(ENTRY, DT, 5) HPRMS_MX_SHAPES(ENTRY, DT, 6) HPRMS_BLOCKQ_SHAPES(ENTRY, DT, 7)
 
 // The shapes with sc1 bits among the lists of modes 0, 1, 3 and 4 (their
 // off-grid variants keep them for calls past the Infinity Cache)
@@ -213,7 +220,7 @@ struct FusedEntry {
   X(DT, MODE, 512, 8, 4, 512, 159) X(DT, MODE, 64, 8, 0, 256, 3) X(DT, MODE, 512, 2, 0, 512, 31)  \
   X(DT, MODE, 512, 4, 0, 512, 31) X(DT, MODE, 512, 8, 0, 512, 7) X(DT, MODE, 1024, 2, 0, 1024, 31) \
   X(DT, MODE, 1024, 3, 0, 1024, 159) X(DT, MODE, 256, 8, 0, 256, 7) X(DT, MODE, 512, 5, 0, 512, 135) \
-  X(DT, MODE, 512, 6, 0, 512, 135)
+  X(DT, MODE, 512, 6, 0, 512, 135) X(DT, MODE, 256, 2, 0, 256, 3) X(DT, MODE, 512, 2, 0, 512, 3)
 
 // The shapes below are built only into the bench library libhprms_bench.so
 // (hprms.hip compiled with HPRMS_BENCH_BUILD), never into libhprms.so: no

@@ -33,3 +33,12 @@ def test_quantised_outputs_at_the_edges_of_their_shapes(ops, rows, hidden, dtype
     test_gpu_fp8_group.run_case(ops, rows, hidden, dtype, seed=hidden + rows)
     test_gpu_mx.run_case(ops, rows, hidden, dtype, oracle.MXFP8, seed=hidden + rows)
     test_gpu_mx.run_case(ops, rows, hidden, dtype, oracle.MXFP4, seed=hidden + rows)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("rows,hidden", [(769, 3200), (768, 4096), (769, 4096), (257, 4224), (257, 5120), (256, 5248),
+                                         (257, 5248), (300, 8064), (4096, 8192)])
+def test_quantised_outputs_with_the_weight_loaded_with_the_row(ops, rows, hidden, dtype):
+    """3K-8K: the first and last widths and the first row counts of the shapes
+    that load the weight early, and the last of those that load it late."""
+    test_quantised_outputs_at_the_edges_of_their_shapes(ops, rows, hidden, dtype)
