@@ -739,11 +739,23 @@ Phase phase8(const void* p, int64_t stride) { return {(uint32_t)((uintptr_t)p & 
 // shifts only rows of odd widths whose streams share one phase (14-34%
 // faster): its byte rows misaligned cost 15-25% at 16K, and for whole-vector
 // widths its unaligned variant was as fast or faster.
+//
+// The partial sums (mode 4) also shift rows of odd widths from 120 whole
+// vectors up when all their streams share one phase: every one of the P + 2
+// streams is off alignment there, and the rows run the tail variant either
+// way.  8 parts, fp16, cold, interleaved trials of one build, at 1001-4097
+// elements: 2-9% faster at 1024 and 2048 rows (0.6% at 1024 x 2503), 4-12% at
+// 3000 and 4096 (4096 x 2503: 12%), 3-14% at 256 rows from 1.5K (256 x 4097:
+// 14%), the same within their spread at 16 rows and at 256 x 1001.  The rule looks
+// at the width alone, so a row's bits do not depend on the call's row count.
 constexpr int64_t kShiftMinVec = 513;
+constexpr int64_t kShiftMinVecParts = 120;
 
 Phase shift_phase(const Problem& p) {
   const Phase none = {0, 0};
-  if (p.mode > 4 || p.hidden / 8 < kShiftMinVec) return none;
+  if (p.mode > 4) return none;
+  const bool narrow = p.hidden / 8 < kShiftMinVec;
+  if (narrow && (p.mode != 4 || p.hidden % 8 == 0 || p.hidden / 8 < kShiftMinVecParts)) return none;
   Phase s[4 + HPRMS_MAX_PARTS];
   int n = 0;
   switch (p.mode) {
@@ -777,7 +789,7 @@ Phase shift_phase(const Problem& p) {
     if (s[i] == none) return none;
     if (!(s[i] == s[0])) shared = false;
   }
-  if (p.mode == 2) return shared && p.hidden % 8 != 0 ? s[0] : none;
+  if (p.mode == 2 || narrow) return shared && p.hidden % 8 != 0 ? s[0] : none;
   if (p.mode == 1 && !shared && p.hidden < 16384) return none;
   return s[0];
 }
