@@ -840,19 +840,24 @@ void fused_vec_kernel(const uint16_t* x_rows,  // input rows (MODE 0: also the o
       }
     } else {
       // y in 16-bit form, kept in the registers x came in, and the row maximum
-      // of |y|.  Slots past the row hold zeros and zero weights: they add a 0,
-      // or a NaN (0 times an infinite or NaN inv) that the row's own elements
-      // give too.  The edge vector's repeated elements are harmless.
+      // of |y| over the row's own elements.  Slots past the row are left out by
+      // a select per vector: they hold zeros, and 0 times an infinite inv (eps 0
+      // and squares that underflow) is NaN, where the row's own y are infinite.
+      // The edge vector's repeated elements are harmless.
       float m = 0.0f;
 #pragma unroll
       for (int k = 0; k < VPL; ++k) {
         const u32x4 s = held(k);
+        float mk = m;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) xv[k][j] = out_pair(s[j], wv[k][j], m);
+        for (int j = 0; j < 4; ++j) xv[k][j] = out_pair(s[j], wv[k][j], mk);
+        m = vec_ok[k] ? mk : m;
       }
       if constexpr (TAIL) {
+        float me = m;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) txv[j] = out_pair(tsv[j], twv[j], m);
+        for (int j = 0; j < 4; ++j) txv[j] = out_pair(tsv[j], twv[j], me);
+        m = eok ? me : m;
       }
       float isc;
       if (has_given) {

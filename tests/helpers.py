@@ -178,6 +178,11 @@ def ulp_neighbours(a):
     return back(o - 1), a.astype(np.uint16), back(o + 1)
 
 
+def _is_nan(y_bits, dtype):
+    """Infinity's upper neighbour is a NaN pattern: no value one ulp away."""
+    return (np.asarray(y_bits, np.uint16) & 0x7FFF) > (0x7F80 if dtype == torch.bfloat16 else 0x7C00)
+
+
 def _e4m3_of(y_bits, isc, dtype):
     with np.errstate(invalid="ignore", over="ignore"):
         v = oracle.to_f32(y_bits, DT[dtype]) * np.asarray(isc, np.float32)
@@ -199,7 +204,8 @@ def assert_fp8_from_y_within_one_ulp(q, y_oracle, isc, dtype, what="q"):
     yi, qi, ii = y[idx], q[idx], isc[idx]
     ok = np.zeros(qi.shape, bool)
     for yc in ulp_neighbours(yi):
-        ok |= oracle.e4m3_ulp_distance(qi, _e4m3_of(yc, ii, dtype)) == 0
+        same = oracle.e4m3_ulp_distance(qi, _e4m3_of(yc, ii, dtype)) == 0
+        ok |= same & (_is_nan(yc, dtype) == _is_nan(yi, dtype))
     bad = np.nonzero(~ok)[0]
     assert bad.size == 0, (f"{what}: {bad.size} elements are no quantisation of a y within 1 ulp; first at "
                            f"{tuple(int(v[bad[0]]) for v in idx)}")
@@ -220,7 +226,8 @@ def assert_group_scales(scales, y_oracle, group, dtype, what="scales"):
         with np.errstate(invalid="ignore"):
             sc = (oracle.to_f32(m & 0x7FFF, DT[dtype]) / np.float32(448.0)).astype(np.float32)
             sc = np.where(sc < tiny, tiny, sc).astype(np.float32)
-        ok |= (got.view(np.uint32) == sc.view(np.uint32)) | (np.isnan(got) & np.isnan(sc))
+        same = (got.view(np.uint32) == sc.view(np.uint32)) | (np.isnan(got) & np.isnan(sc))
+        ok |= same & (_is_nan(m, dtype) == _is_nan(mag, dtype))
     bad = np.argwhere(~ok)
     assert bad.size == 0, f"{what}: {len(bad)} scales off; first {bad[0]}: {got[tuple(bad[0])]}"
 

@@ -107,6 +107,35 @@ def test_fp8_ub_special_rows_and_bounds(ops):
             run_case(ops, rows, hidden, torch.bfloat16, rows + hidden, ub, special=True)
 
 
+# widths whose rows leave lanes idle, of every FP8 table row and the tail
+# variants (odd widths: most lanes hold no edge vector), and one that leaves none
+@pytest.mark.parametrize("hidden", [1000, 1024, 1800, 2056, 3200, 5000, 5120, 9000, 13000, 17000, 22000, 25000,
+                                    1001, 3201, 4097, 13313, 16391, 20481, 24697])
+@pytest.mark.parametrize("rows", [5, 1100])
+def test_fp8_rows_whose_squares_underflow_without_eps(ops, rows, hidden):
+    """eps = 0 and rows whose squares are all zero in binary32: inv and every
+    y are infinite, and so is the row maximum, whatever the width; a bound
+    makes the scale finite and every code the largest finite one."""
+    print("fp8 underflowing rows", rows, hidden, flush=True)
+    x, r, w = make_inputs(rows, hidden, torch.bfloat16, hidden)
+    x = torch.sign(x)
+    x[x == 0] = 1.0
+    tiny = torch.tensor([1e-25, 1e-39, 1e-30])[torch.arange(rows) % 3]
+    x, r = (x * tiny[:, None]).to(torch.bfloat16), torch.zeros_like(r)
+    th = min(16, oracle.max_threads())
+    for ub in (float("nan"), 4.0):
+        oq, osc, ores = oracle.fused_add_rmsnorm_fp8_ub(bits(x), bits(w), bits(r), 0.0, oracle.BF16, ub, threads=th)
+        assert (osc == (np.float32(4.0) / np.float32(448.0) if ub == 4.0 else np.inf)).all()
+        for bounded in ((True,) if ub == 4.0 else (True, False)):
+            rd = r.to(DEV)
+            ubd = torch.tensor([ub], dtype=torch.float32, device=DEV) if bounded else None
+            q, sc = ops.fused_add_rms_norm_fp8(x.to(DEV), rd, w.to(DEV), 0.0, scale_ub=ubd)
+            torch.cuda.synchronize()
+            assert same_floats(sc.reshape(-1).cpu().numpy(), osc), (rows, hidden, ub, bounded, sc.reshape(-1)[:3])
+            assert oracle.e4m3_ulp_distance(q_bits(q), oq).max() == 0, (rows, hidden, ub, bounded)
+            assert_residual_exact(bits(rd), ores, torch.bfloat16)
+
+
 def test_fp8_ub_through_the_c_abi_and_its_checks(ops):
     from hp_rms_norm_amd import abi
     rows, hidden = 64, 4096

@@ -440,6 +440,28 @@ def test_oracle_fp8_static_quantisation_matches_torch():
                 assert d.max() == 0, (code, kind, scale)
 
 
+def test_fp8_checks_tell_nan_from_infinity():
+    """The FP8 parity checks allow a neighbouring 16-bit value, but a NaN scale
+    or code only where the oracle's y is NaN: infinity's upper neighbour is a
+    NaN pattern, and a NaN pattern's lower neighbour may be infinity."""
+    from helpers import assert_fp8_from_y_within_one_ulp, assert_group_scales
+    for code in (BF, HF):
+        dt = TDT[code]
+        inf, one, nan = (0x7F80, 0x3F80, 0x7F81) if code == BF else (0x7C00, 0x3C00, 0x7C01)
+        y = np.array([[inf, one, one, one]], np.uint16)
+        assert_group_scales(np.array([np.inf], np.float32), y, 4, dt)
+        with pytest.raises(AssertionError):
+            assert_group_scales(np.array([np.nan], np.float32), y, 4, dt)
+        y[0, 0] = nan
+        assert_group_scales(np.array([np.nan], np.float32), y, 4, dt)
+        with pytest.raises(AssertionError):
+            assert_group_scales(np.array([np.inf], np.float32), y, 4, dt)
+        y = np.array([[inf]], np.uint16)
+        assert_fp8_from_y_within_one_ulp(np.array([[0x7E]], np.uint8), y, np.float32(1.0), dt)
+        with pytest.raises(AssertionError):
+            assert_fp8_from_y_within_one_ulp(np.array([[0x7F]], np.uint8), y, np.float32(1.0), dt)
+
+
 def test_oracle_fp8_static_and_group_match_golden(golden):
     """The torch-made golden vectors of the static and per-group FP8 forms: the
     residual bit-exact; where the oracle's 16-bit output equals torch's (every
