@@ -746,8 +746,12 @@ Phase phase8(const void* p, int64_t stride) { return {(uint32_t)((uintptr_t)p & 
 // way.  8 parts, fp16, cold, interleaved trials of one build, at 1001-4097
 // elements: 2-9% faster at 1024 and 2048 rows (0.6% at 1024 x 2503), 4-12% at
 // 3000 and 4096 (4096 x 2503: 12%), 3-14% at 256 rows from 1.5K (256 x 4097:
-// 14%), the same within their spread at 16 rows and at 256 x 1001.  The rule looks
-// at the width alone, so a row's bits do not depend on the call's row count.
+// 14%), the same within their spread at 16 rows and at 256 x 1001.  With parts
+// at other phases than the output's and the residual's, shifting ranged from
+// 5.5% faster to 7% slower (2 parts, 1025 x 4097), so the rows stay unshifted.
+// Where the parts are slices of one buffer their phases follow from the row
+// count (slice g of [parts, rows, H] starts g * rows * H elements in), and with
+// them a row's summation order: in batch-invariant mode no narrow row is shifted.
 constexpr int64_t kShiftMinVec = 513;
 constexpr int64_t kShiftMinVecParts = 120;
 
@@ -755,7 +759,8 @@ Phase shift_phase(const Problem& p) {
   const Phase none = {0, 0};
   if (p.mode > 4) return none;
   const bool narrow = p.hidden / 8 < kShiftMinVec;
-  if (narrow && (p.mode != 4 || p.hidden % 8 == 0 || p.hidden / 8 < kShiftMinVecParts)) return none;
+  if (narrow && (p.mode != 4 || p.hidden % 8 == 0 || p.hidden / 8 < kShiftMinVecParts || batch_invariant()))
+    return none;
   Phase s[4 + HPRMS_MAX_PARTS];
   int n = 0;
   switch (p.mode) {

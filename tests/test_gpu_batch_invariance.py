@@ -135,3 +135,31 @@ def test_other_forms_do_not_depend_on_the_row_count(abi, invariant, form):
             for k, (a, b) in enumerate(zip(run(rows), full)):
                 assert np.array_equal(a, b[: a.shape[0]]), f"{form}: output {k}, {rows} rows x {hidden}"
 
+
+
+# odd widths below 513 whole vectors (and one above): the partial sums may be
+# shifted onto the streams' shared phase
+@pytest.mark.parametrize("hidden", [961, 1501, 2503, 4097, 4111])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_partial_sums_of_one_buffer_do_not_depend_on_the_row_count(abi, invariant, hidden, dtype):
+    """Parts that are slices of one [parts, rows, H] buffer: slice g starts
+    g * rows * H elements in, so for an odd H the row count sets the parts'
+    alignment relative to the output's."""
+    total, code = 1032, DT[dtype]
+    print(f"stacked parts x {hidden} {dtype}", flush=True)
+    for nparts in (2, 8):
+        p, r, w = make_inputs(nparts * total, hidden, dtype, seed=hidden + nparts)
+        p, r, wd = p.view(nparts, total, hidden), r[:total], w.to(DEV)
+
+        def run(n):
+            pd, rd = p[:, :n].contiguous().to(DEV), r[:n].to(DEV)
+            od = torch.empty((n, hidden), dtype=dtype, device=DEV)
+            abi.reduce_add_rmsnorm(od.data_ptr(), [t.data_ptr() for t in pd], wd.data_ptr(), rd.data_ptr(), n, hidden,
+                                   hidden, hidden, hidden, code, 1e-6, _stream())
+            torch.cuda.synchronize()
+            return bits(od), bits(rd)
+
+        full = run(total)
+        for rows in (8, 9, 64, 65, 256, 257, 1024, 1025, 1030):
+            for k, (a, b) in enumerate(zip(run(rows), full)):
+                assert np.array_equal(a, b[:rows]), f"output {k}, {nparts} parts, {rows} rows x {hidden}"
