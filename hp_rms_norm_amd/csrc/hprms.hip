@@ -227,6 +227,10 @@ bool latency_config(int64_t rows, int64_t nvec, int mode, hprms_config* c) {
 // 4096.  Past 24K the LDS tier (per row) and 1024 x 4 (per block) stay, 2-5%
 // ahead of 512 x 8 in registers.  256 x 8 against 512 x 4 at 16384: MXFP4
 // 2-4% and FP8 per 128 elements 2% faster, per-row FP8 the same.
+// Only there: at 14464-16128 columns 512 x 4 is 1-3% faster than 256 x 8 from
+// 1024 rows (15360 columns, MXFP8: 4096 rows 75.2 -> 74.4 us), 2-8% at 300 rows
+// and 1-5% with 512-1024 rows resident; it is 1.5-3% slower at 512 rows, cold,
+// and the same off the 128-byte grid and at 64 rows.
 // 256 x 2 and 512 x 2 load the weight with the row (flags 3) in the per-row
 // FP8 and MX forms: their output phase is long enough that a weight load
 // issued after the residual's stores is waited for with nothing else to do.
@@ -247,9 +251,8 @@ bool quant_config(int64_t nvec, int mode, bool grid, hprms_config* c) {
                        {all, 513, 640, 256, 3, 0, 256, 7},
                        {early, 641, 1024, 512, 2, 0, 512, 3},
                        {all, 641, 1024, 512, 2, 0, 512, 7},
-                       {row, 1537, 2048, 512, 4, 0, 512, 7},
-                       {blocks, 1537, 1792, 512, 4, 0, 512, 7},
-                       {blocks, 1793, 2048, 256, 8, 0, 256, 7},
+                       {blocks, 2048, 2048, 256, 8, 0, 256, 7},
+                       {all, 1537, 2048, 512, 4, 0, 512, 7},
                        {all, 2049, 2560, 512, 5, 0, 512, 135},
                        {all, 2561, 3072, 512, 6, 0, 512, 135},
                        {row, 3073, 4096, 512, 8, 4, 512, 159},

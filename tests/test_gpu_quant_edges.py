@@ -21,7 +21,7 @@ def ops():
     return hp_rms_norm_amd
 
 
-WIDTHS = [12416, 14336, 14464, 16512, 20480, 20608, 24704]
+WIDTHS = [12416, 14336, 14464, 16256, 16384, 16512, 20480, 20608, 24704]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
