@@ -155,20 +155,11 @@ __device__ __forceinline__ void store1(uint8_t v, __amdgpu_buffer_rsrc_t r, uint
 }
 
 // ---- OCP MX (E2M1 elements) ----------------------------------------------------------
-// Two binary32 values to two E2M1 codes in byte SEL of w, the first value in
-// the low nibble (gfx950 v_cvt_scalef32_pk_fp4_f32 with scale 1.0: round to
-// nearest even, saturating at +-6; NaN gives code 7 with NaN's sign).  The
-// other bytes of w are kept.
-template <int SEL>
-__device__ __forceinline__ uint32_t cvt_e2m1x2(uint32_t w, float a, float b) {
-  return __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, a, b, 1.0f, SEL);
-}
-
-// The same from two packed 16-bit values, each divided by `scale` (a power of
-// two given by its exponent field alone: 0 stands for 2^-127), and two e4m3fn
-// bytes in half HI of w likewise (overflow gives code 0x7f).  Every 16-bit
-// value at every scale byte 0-253 measured the same code as the binary32
-// product's conversion.
+// Two packed 16-bit values, each divided by `scale` (a power of two given by
+// its exponent field alone: 0 stands for 2^-127), to two E2M1 codes in byte
+// SEL of w, the first value in the low nibble (gfx950
+// v_cvt_scalef32_pk_fp4_bf16 / _f16: round to nearest even, saturating at
+// +-6); the other bytes of w are kept.
 template <int DT, int SEL>
 __device__ __forceinline__ uint32_t cvt_scaled_e2m1x2(uint32_t w, uint32_t y, float scale) {
   if constexpr (DT == HPRMS_DTYPE_BF16)
@@ -177,6 +168,8 @@ __device__ __forceinline__ uint32_t cvt_scaled_e2m1x2(uint32_t w, uint32_t y, fl
     return __builtin_amdgcn_cvt_scalef32_pk_fp4_f16(w, __builtin_bit_cast(f16x2, y), scale, SEL);
 }
 
+// The same to two e4m3fn bytes in half HI of w (v_cvt_scalef32_pk_fp8_bf16 /
+// _f16; past 464 the overflow code 0x7f).
 typedef short s16x2 __attribute__((ext_vector_type(2)));
 template <int DT, bool HI>
 __device__ __forceinline__ uint32_t cvt_scaled_e4m3x2(uint32_t w, uint32_t y, float scale) {
