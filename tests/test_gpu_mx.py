@@ -113,6 +113,44 @@ def test_mx_blocks_across_the_exponent_range(ops, dtype, fmt):
         assert np.all(sc[:, 0] == 0) and sc[:, 1].min() >= (230 if fmt == "mxfp8" else 236)
 
 
+def every_value_below_every_block_maximum(dtype):
+    """16-bit patterns in blocks of 32: for each exponent of the type (fp16:
+    and each subnormal magnitude), every value of either sign not above the
+    largest value with it, in blocks that start with that largest value."""
+    if dtype == torch.bfloat16:
+        tops = [(e << 7) | 0x7F for e in range(255)]
+    else:
+        tops = [(1 << k) - 1 for k in range(1, 11)] + [(e << 10) | 0x3FF for e in range(1, 31)]
+    blocks = []
+    for top in tops:
+        mag = np.arange(top + 1, dtype=np.uint32)
+        v = np.concatenate([mag, mag | 0x8000]).astype(np.uint16)
+        v = np.concatenate([v, np.zeros(-len(v) % 31, np.uint16)]).reshape(-1, 31)
+        blocks.append(np.concatenate([np.full((len(v), 1), top, np.uint16), v], axis=1))
+    return np.concatenate(blocks)
+
+
+@pytest.mark.parametrize("fmt", sorted(FMT))
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_mx_every_value_at_every_block_scale(ops, dtype, fmt):
+    """The conversions' scale operand, rounding, saturation and subnormals: a
+    row of ones with eps = 0 has the inverse 1, so y is the weight itself, and
+    the weight carries every 16-bit value at every scale a block of it gets."""
+    blocks = every_value_below_every_block_maximum(dtype)
+    hidden = 65536
+    y = np.concatenate([blocks.reshape(-1), np.zeros(-blocks.size % hidden, np.uint16)]).reshape(-1, hidden)
+    print("mx every value", fmt, dtype, y.shape, flush=True)
+    wd = torch.from_numpy(y.view(np.int16)).to(DEV).view(dtype)
+    one = torch.ones((1, hidden), dtype=dtype, device=DEV)
+    fn = ops.fused_add_rms_norm_mxfp8 if fmt == "mxfp8" else ops.fused_add_rms_norm_mxfp4
+    got = [fn(one, torch.zeros_like(one), wd[i], 0.0) for i in range(len(y))]
+    torch.cuda.synchronize()
+    q, sc = (np.concatenate([u8(g[k]) for g in got]) for k in (0, 1))
+    wq, wsc = oracle.mx_quantize(y, DT[dtype], FMT[fmt])
+    assert wsc.max() < 0xFF and len(np.unique(wsc)) >= (245 if dtype == torch.bfloat16 else 30)
+    compare_blocks(q, sc, wq, wsc, hidden, FMT[fmt], f"every value {fmt} {dtype}")
+
+
 @pytest.mark.parametrize("fmt", sorted(FMT))
 def test_mx_zero_nan_and_huge_rows(ops, fmt):
     rows, hidden, dtype = 8, 1024, torch.bfloat16
