@@ -181,7 +181,9 @@ int64_t rows_at_ref(int64_t rows, int cus) {
 // loaded together with the row: a one- or two-wave row then waits for one
 // memory round trip instead of two (H = 1024: 2.4-4.5% faster for the fused,
 // out-of-place and MX forms, 1-256 rows, hot and cold; H = 2048: up to 1.2%).
-// From 4096 up, loading it after the row's sum measured as fast or faster.
+// From 4096 up, loading it after the row's sum measured as fast or faster in
+// the 16-bit op, and the other forms' latency rows follow it (not measured
+// there for the quantised outputs).
 //
 // These rows stay ahead of the bandwidth table well past one row per CU, by
 // how much depending on the mode, so the largest row count that still takes
@@ -220,13 +222,18 @@ bool latency_config(int64_t rows, int64_t nvec, int mode, hprms_config* c) {
 // table's 64 x 4 at 4096 rows), 256 lanes x 2 at 3K < H <= 4K, and from 12K
 // on workgroups of 256 and 512 lanes with more vectors each rather than 1024
 // lanes: more workgroups stand on a CU, so the barriers of one hide behind
-// the loads of others.  Against 1024 x 2 at 16384 (bf16; per-row FP8, MXFP4):
-// 512 rows 13.7 -> 11.9 us and 12.4 -> 10.8 us, 4096 rows 83.0 -> 78.8 us and
-// 75.3 -> 71.6 us; 512 x 5-6 against 1024 x 3: per-row FP8 11-30% faster at
-// 20K-24K from 1 to 4096 rows, MXFP4 4-23% up to 768 rows and within 2% at
-// 4096.  Past 24K the LDS tier (per row) and 1024 x 4 (per block) stay, 2-5%
-// ahead of 512 x 8 in registers.  256 x 8 against 512 x 4 at 16384: MXFP4
-// 2-4% and FP8 per 128 elements 2% faster, per-row FP8 the same.
+// the loads of others.  Against 1024 x 2 at 16384 (bf16; per-row FP8, MXFP4),
+// with the same output phase: 512 rows 13.7 -> 11.9 us and 12.4 -> 10.8 us,
+// 4096 rows 83.0 -> 78.8 us and 75.3 -> 71.6 us; 512 x 5-6 against 1024 x 3
+// at 16.5K-24.5K, MX: 1-15% faster from 512 to 8192 rows (off the 128-byte grid
+// at 24576: 0-3% slower).  Against the library as it was before the output
+// phase was shortened, per-row FP8 and FP8 per 128 elements take 7-30% less
+// time at 16.5K-24.5K, MX 14-26% at one row and 2-10% at 300-512; from 1536
+// rows MX ranges from 4% faster to 1.7% slower in 512 x 5 and is 0.5-2.8%
+// slower at 22.5K-24.5K in 512 x 6 (4096 x 24576 MXFP8: 116.0 -> 117.7 us).  Past 24K
+// the LDS tier (per row) and 1024 x 4 (per block) stay, 2-5% ahead of 512 x 8
+// in registers.  256 x 8 against 512 x 4 at 16384: MXFP4 2-4% and FP8 per 128
+// elements 2% faster, per-row FP8 the same.
 // Only there: at 14464-16128 columns 512 x 4 is 1-3% faster than 256 x 8 from
 // 1024 rows (15360 columns, MXFP8: 4096 rows 75.2 -> 74.4 us), 2-8% at 300 rows
 // and 1-5% with 512-1024 rows resident; it is 1.5-3% slower at 512 rows, cold,
@@ -237,7 +244,9 @@ bool latency_config(int64_t rows, int64_t nvec, int mode, hprms_config* c) {
 // Cold, interleaved trials, bf16, H = 3584-8192 at 1024 / 2048 / 4096 / 8192
 // rows: per-row FP8 2.0-4.0 / 1.4-3.6 / 0.2-1.7 / up to 1.3% faster (2048 x
 // 8192: 21.8 -> 21.5 us), MXFP8 1.4-5.6 / 1.2-4.9 / 0-2.1 / within 0.9%,
-// MXFP4 1.3-7.2 / 2.3-4.0 / 0.5-1.4 / within 0.6%.  Per-row FP8 keeps the late
+// MXFP4 1.3-7.2 / 2.3-4.0 / 0.5-1.4 / within 0.6%.  With the rows resident in
+// the Infinity Cache the late weight is 2-4% faster (5K-8K, 300-2048 rows), so
+// MX calls of 1024 x 6144-8192 on such rows lost 2-5%.  Per-row FP8 keeps the late
 // weight off the 128-byte grid (`grid`: its tail variant holds an edge vector
 // too); so do 256 x 3 (early: MX 4% faster at 1024 rows, 1.5% slower at 8192,
 // FP8 3.5% faster to 1.3% slower) and FP8 per 128 elements.
@@ -318,9 +327,9 @@ bool reduce_config(int64_t nvec, hprms_config* c) {
 // together with the row in the fused op and its out-of-place and partial-sum
 // forms (modes 0, 3, 4): 0.8-1.6% faster (bf16 and fp16, on the 128-byte grid
 // and rotated off it; 4096 rows, two builds side by side, 9 interleaved
-// trials; one row: 2% slower).  Plain RMSNorm measured the same either way;
-// the FP8 and MX outputs ran 12-23% slower with it and the tail variants
-// 2-4% (tail_shape): they load it late.
+// trials; one row: 2% slower).  Plain RMSNorm, the only other form with these
+// shapes, measured the same either way and the tail variants 2-4% slower with
+// it (tail_shape): they load it late.
 bool weight_late_1024(int mode, const hprms_config& c) {
   if (c.lanes_per_row != 1024 || (c.vec_per_lane != 2 && c.vec_per_lane != 3)) return false;
   return !(mode == 0 || mode == 3 || mode == 4);
@@ -473,8 +482,9 @@ void table_config(int64_t rows, int64_t hidden, int mode, bool grid, int cus, hp
 // 2.3 / 3.7 / 3.0%, 4096 2.3 / 2.4 / 2.8 / 2.6%, 8192 2.3 / 3.1 / 5.6 / 2.2%;
 // at 512 rows -1% to +3.7%: left out).  With rows of scales mode 7 ranged from
 // 1.1% faster to 0.6% slower, and at 8 KiB rows modes 2, 5 and 6 were within
-// 0.4% either way, so left out.  At 32 and 64 KiB rows (1024 lanes, one row
-// per workgroup) runs of 8-64 were 3-13% slower in mode 7.
+// 0.4% either way, so left out.  In mode 7 runs of 32 were 1% slower (rows of
+// scales) and 1% faster (columns) at 32 KiB rows (256 x 8), and 2-5% slower
+// at 64 KiB (1024 x 4).
 struct RunsRow {
   unsigned modes;       // bit m: mode m
   bool scale_columns;   // mode 7 with column-major scales only
@@ -746,10 +756,11 @@ Phase phase8(const void* p, int64_t stride) { return {(uint32_t)((uintptr_t)p & 
 // The partial sums (mode 4) also shift rows of odd widths from 120 whole
 // vectors up when all their streams share one phase: every one of the P + 2
 // streams is off alignment there, and the rows run the tail variant either
-// way.  8 parts, fp16, cold, interleaved trials of one build, at 1001-4097
-// elements: 2-9% faster at 1024 and 2048 rows (0.6% at 1024 x 2503), 4-12% at
-// 3000 and 4096 (4096 x 2503: 12%), 3-14% at 256 rows from 1.5K (256 x 4097:
-// 14%), the same within their spread at 16 rows and at 256 x 1001.  With parts
+// way.  fp16, cold, interleaved trials, 961-4097 elements, 8 parts: 0-5% faster
+// at 1024 rows, 3-8% at 2048, 3-10% at 3000 and 4096 (4096 x 2503: 43.9 ->
+// 39.6 us), 4-15% at 256 rows from 1.5K (256 x 4097: 8.0 -> 6.8 us), 1-22% at
+// 16 rows.  2 and 4 parts: 2-12% faster from 2048 rows (1% at 3000 x 2001), 1%
+// slower to 8% faster at 1024, up to 2.5% slower at 16 rows below 1.5K.  With parts
 // at other phases than the output's and the residual's, shifting ranged from
 // 5.5% faster to 7% slower (2 parts, 1025 x 4097), so the rows stay unshifted.
 // Where the parts are slices of one buffer their phases follow from the row

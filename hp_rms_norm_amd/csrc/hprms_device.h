@@ -118,9 +118,10 @@ struct Fmt<HPRMS_DTYPE_FP16> {
 // ---- FP8 ----------------------------------------------------------------------
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-// Four binary32 values to four OCP e4m3fn bytes (gfx950 v_cvt_pk_fp8_f32:
-// round to nearest even; callers clamp to +-448 first).  Byte i of the result
-// holds value i.
+// Four binary32 values, each NaN or at most 464 in magnitude, to four OCP
+// e4m3fn bytes (gfx950 v_cvt_pk_fp8_f32: round to nearest even, so 448-464
+// gives 448; callers clamp what can pass 464).  Byte i of the result holds
+// value i.
 __device__ __forceinline__ uint32_t pack_e4m3x4(float a, float b, float c, float d) {
   int w = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false);
   w = __builtin_amdgcn_cvt_pk_fp8_f32(c, d, w, true);

@@ -77,8 +77,9 @@
 // (1 / scale))) to q), or, with FusedArgs::static_scale set, with that one
 // given scale for every row (no row maximum, no scale written); the residual
 // is updated in place and `input` is only read.
-// The row maximum is a second DPP/LDS reduction over the 16-bit magnitudes
-// (sign-magnitude bit patterns order like their values, NaN above inf).
+// The row maximum is a second DPP/LDS reduction over the magnitudes of the
+// binary32 products that y is rounded from (their bit patterns order like
+// their values, NaN above inf); rounded once, it is the maximum of |y|.
 // MODE 3 is the fused op out of place: input and residual are only read, the
 // sum goes to res_out and the output to out.  MODE 4 adds nparts partial rows
 // first (the buffers of a tensor-parallel all-reduce): a = rne(p0 + p1 + ...)
@@ -209,8 +210,7 @@ void fused_vec_kernel(const uint16_t* x_rows,  // input rows (MODE 0: also the o
   constexpr uint32_t CH = LPR * 16;  // byte distance between a lane's vectors
   // FLAGS bit 10 (bench library): row groups in xcd_xor's order; bits 16-18,
   // V > 0: in xcd_runs<V>'s order (runs of 2^V row groups per XCD; the table
-  // takes it for the in-place op at two row pitches, the bench library for
-  // its sweeps)
+  // takes it where hprms.hip's kRuns says, the bench library for its sweeps)
   constexpr bool WXOR = (FLAGS & 1024) != 0;
   constexpr int WRUNS = (FLAGS >> 16) & 7;
   // The output phase's unpack of the held row.  With the square phase's lo /

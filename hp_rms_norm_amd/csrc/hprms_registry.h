@@ -28,7 +28,7 @@ struct FusedEntry {
 // the stores (bench library), bit 14 = the tail variant's weight staged in
 // LDS, bit 15 = the partial sums' parts loaded before any is added, bits
 // 16-18 = V > 0: row groups in runs of 2^V per XCD (xcd_runs; the product
-// has two, hprms.hip kRuns),
+// has those of hprms.hip's kRuns),
 // bit 19 = the output phase at raised wave priority (bench library), bits 20
 // / 21 = the two load orders alternating per wave / per workgroup (with bit 7;
 // bench library)
