@@ -1,8 +1,8 @@
 """Benchmark of the fused residual-add + RMSNorm path on one MI355X.
 
-Workload (BASELINE.json's metric): bf16 fused add+RMSNorm at (4096, H) for
-every H of configs[1] (1024 ... 12288 step 1024) and configs[2] (13312 ...
-32768).  One step = one call at each of those H, in order.  Inputs are
+Workload: bf16 fused add+RMSNorm at (4096, H) for every H of 1024 ... 12288
+step 1024 and of 13312, 14336, 16384, 20480, 24576, 28672 and 32768.  One step
+= one call at each of those H, in order.  Inputs are
 resident in HBM before timing starts; every H has two buffer sets used
 alternately, and one step moves ~3.8 GB, so no call finds its rows in the
 256 MB Infinity Cache left over from its previous use.
@@ -24,8 +24,8 @@ cpu_baseline = the reference's CPU path: its test's torch formula
 cpu_oracle   = the CPU oracle (a scalar C restatement, OpenMP over rows) on a
                bounded sample of the same shapes.
 details    = printed before the bench line, one JSON line per section
-             ({"bench_detail": name, "data": ...}): BASELINE.json's other
-             configs (decode, fp16, streamer) and the other operators (FP8 /
+             ({"bench_detail": name, "data": ...}): the other
+             workloads (decode, fp16, streamer) and the other operators (FP8 /
              MX outputs, out-of-place, plain RMSNorm, rows off the 128-byte
              grid, partial sums), µs/call; a copy moving the fused op's bytes
              at six of the widths, with the fused op's time as a fraction of
@@ -1077,10 +1077,10 @@ def load_traffic(key):
 
 
 def run_extra(torch, ops, args):
-    """BASELINE.json's other configs, µs/call (median over timed calls)."""
+    """The other workloads, µs/call (median over timed calls)."""
     out = {}
     steps = max(10, args.steps)
-    # configs[3]: decode shapes with 1% outliers x50
+    # decode shapes with 1% outliers x50
     dec = [(b, h, torch.bfloat16, "outliers") for b in (1, 8, 32, 128, 512) for h in (4096, 8192)]
     us = time_shapes(torch, ops.hp_rms_norm, dec, steps, args.warmup)
     out["decode_bf16"] = [{"rows": b, "hidden": h, "us_per_call": round(u, 2), "us_p10": round(p10, 2),
@@ -1129,7 +1129,7 @@ def run_extra(torch, ops, args):
     out["batch_invariant_mode_bf16"] = [
         {"rows": b, "hidden": h, "us_per_call": round(u, 2), "default_mode_us_per_call": round(default_us[(b, h)], 2)}
         for (b, h, _, _), (u, _, _) in zip(dec + mid, inv)]
-    # configs[4]: fp16 non-power-of-two hidden
+    # fp16 non-power-of-two hidden
     f16 = [(B, 5120, torch.float16, "bench"), (B, 7168, torch.float16, "bench")]
     us = time_shapes(torch, ops.hp_rms_norm, f16, steps, args.warmup)
     out["fp16"] = [{"rows": b, "hidden": h, "us_per_call": round(u, 2), "us_p10": round(p10, 2),
@@ -1329,7 +1329,7 @@ def run_extra(torch, ops, args):
                 redd.append({"parts": nparts, "rows": rows, "hidden": h, "us_per_call": round(us, 2)})
                 del sets
     out["reduce_parts_decode_bf16"] = redd
-    # configs[4]: streamer (the reference "relu" = copy, and the true ReLU) at (4096, 14336)
+    # streamer (the reference "relu" = copy, and the true ReLU) at (4096, 14336)
     rows, h = B, 14336
     res = []
     for dtype in (torch.bfloat16, torch.float16):
